@@ -528,6 +528,20 @@ def norm_gate(x, gate, weight, out, eps, device) -> None:
     _check(entry, getattr(lib, entry)(ctypes.byref(args), stream))
 
 
+def _expect(op, name, x, dtype, device, shape, wider=False) -> None:
+    """What a kernel that is handed x's address relies on: its dtype, its device (a GPU) and its shape, contiguous (with
+    `wider`, rows of unit stride that may be longer)."""
+    fits = x.dim() == len(shape) and x.shape[-1] >= shape[-1] and x.shape[:-1] == shape[:-1] if wider else \
+        tuple(x.shape) == shape
+    if not fits or x.dtype != dtype:
+        raise ValueError(f"{op}: {name} must be {dtype} {list(shape)}{' or wider' if wider else ''}, got {x.dtype} "
+                         f"{list(x.shape)}")
+    if not (x.stride(-1) == 1 or x.shape[-1] == 1 if wider else x.is_contiguous()):
+        raise ValueError(f"{op}: {name} must be contiguous")
+    if not x.is_cuda or x.device != device:
+        raise ValueError(f"{op}: all tensors must be on one GPU")
+
+
 def add_norm(residual, add, weight, eps, total, out) -> None:
     """Enqueue gdr_add_norm_fwd on torch's current stream: total = residual + add, out = rmsnorm(total) * weight over
     contiguous [rows, dim] tensors; add, total and out may be None."""
@@ -561,7 +575,10 @@ def head_norm(x, q_heads, k_heads, head_dim, q_weight, k_weight, eps) -> None:
 
 
 def swiglu(gate_up, out) -> None:
-    """Enqueue gdr_swiglu_fwd on torch's current stream: out = silu(gate) * up for the halves of gate_up [T, 2 I]."""
+    """Enqueue gdr_swiglu_fwd on torch's current stream: out = silu(gate) * up for the first and second I columns of
+    gate_up [T, >= 2 I], out [T, I] contiguous, both bf16."""
+    _expect("swiglu", "gate_up", gate_up, torch.bfloat16, out.device, (out.shape[0], 2 * out.shape[-1]), wider=True)
+    _expect("swiglu", "out", out, torch.bfloat16, out.device, (out.shape[0], out.shape[-1]))
     args = GdrSwigluArgs()
     args.abi_version = ABI_VERSION
     args.rows, args.dim = out.shape

@@ -108,3 +108,27 @@ def test_replaced_weights_and_hidden_dtypes():
     half, _ = model.forward(hidden.half(), cu)
     ref, _ = model.forward(hidden.half().float(), cu)
     assert torch.equal(half, ref)
+
+
+def _small_stack():
+    """A KDA and an attention layer, and inputs for them."""
+    cfg = stack.StackConfig(hidden_size=128, intermediate_size=96, num_layers=2, num_attention_heads=2,
+                            num_key_value_heads=1, head_dim=64, kda_num_heads=2, kda_head_dim=64, attention_interval=2)
+    cu = torch.tensor([0, 40, 70], dtype=torch.int32, device="cuda")
+    return stack.HybridStack(cfg, stack.init_weights(cfg, seed=1)), _rand(1, 70, 128, seed=12), cu
+
+
+def test_mlp_weights_of_other_sizes():
+    """An `up` narrower than `gate` is refused as PyTorch's product refuses it; a single gate row broadcasts."""
+    model, hidden, cu = _small_stack()
+    w = model.layers[1]
+    up, gate = w["up"], w["gate"]
+    w["up"] = up[:64].clone()
+    with pytest.raises(RuntimeError):
+        model.forward(hidden, cu)
+    w["up"], w["gate"] = up, gate[:1].clone()
+    one, _ = model.forward(hidden, cu)
+    w["gate"] = gate[:1].expand(96, 128).contiguous()
+    full, _ = model.forward(hidden, cu)
+    # silu(gate) rounded to bf16 in between, or not: 2^-8 of the MLP's share of the stream
+    assert (one - full).norm() <= 2.0 ** -8 * (full - hidden).norm()

@@ -422,3 +422,16 @@ def test_integration_stub_builds_args_the_library_accepts():
         own = lib.make_args(lib.KDA, q, k, v, g, beta, o, K ** -0.5, None, None)
         want = lib.load_library().gdr_chunk_workspace_bytes(ctypes.byref(own))
         assert got == want > 0, (got, want, ns["lib"].gdr_last_error())
+
+
+def test_swiglu_wrapper_checks_shapes_before_any_pointer():
+    out = torch.empty(5, 96, dtype=torch.bfloat16)
+    for shape in ((5, 160), (4, 192), (5, 192, 1)):  # too narrow for two halves, too few rows, another rank
+        with pytest.raises(ValueError, match="gate_up"):
+            lib.swiglu(torch.empty(shape, dtype=torch.bfloat16), out)
+    with pytest.raises(ValueError, match="gate_up"):
+        lib.swiglu(torch.empty(5, 192, dtype=torch.float16), out)
+    with pytest.raises(ValueError, match="contiguous"):
+        lib.swiglu(torch.empty(192, 5, dtype=torch.bfloat16).t(), out)
+    with pytest.raises(ValueError, match="GPU"):
+        lib.swiglu(torch.empty(5, 192, dtype=torch.bfloat16), out)
