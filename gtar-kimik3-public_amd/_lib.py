@@ -528,9 +528,9 @@ def norm_gate(x, gate, weight, out, eps, device) -> None:
     _check(entry, getattr(lib, entry)(ctypes.byref(args), stream))
 
 
-def _expect(op, name, x, dtype, device, shape, wider=False) -> None:
-    """What a kernel that is handed x's address relies on: its dtype, its device (a GPU) and its shape, contiguous (with
-    `wider`, rows of unit stride that may be longer)."""
+def _expect(op, name, x, dtype, shape, wider=False) -> None:
+    """What a kernel that is handed x's address relies on: its dtype and shape, contiguous (with `wider`, rows of unit
+    stride that may be longer)."""
     fits = x.dim() == len(shape) and x.shape[-1] >= shape[-1] and x.shape[:-1] == shape[:-1] if wider else \
         tuple(x.shape) == shape
     if not fits or x.dtype != dtype:
@@ -538,7 +538,10 @@ def _expect(op, name, x, dtype, device, shape, wider=False) -> None:
                          f"{list(x.shape)}")
     if not (x.stride(-1) == 1 or x.shape[-1] == 1 if wider else x.is_contiguous()):
         raise ValueError(f"{op}: {name} must be contiguous")
-    if not x.is_cuda or x.device != device:
+
+
+def _expect_one_gpu(op, *tensors) -> None:
+    if any(t is not None and (not t.is_cuda or t.device != tensors[0].device) for t in tensors):
         raise ValueError(f"{op}: all tensors must be on one GPU")
 
 
@@ -563,6 +566,11 @@ def add_norm(residual, add, weight, eps, total, out) -> None:
 def head_norm(x, q_heads, k_heads, head_dim, q_weight, k_weight, eps) -> None:
     """Enqueue gdr_head_norm_fwd on torch's current stream: the heads of the rows of x [T, >= (q + k) heads * D], in
     place."""
+    heads = q_heads + k_heads
+    _expect("head_norm", "x", x, torch.bfloat16, (x.shape[0], heads * head_dim), wider=True)
+    for name, w in (("q_weight", q_weight), ("k_weight", k_weight)):
+        _expect("head_norm", name, w, torch.float32, (head_dim,))
+    _expect_one_gpu("head_norm", x, q_weight, k_weight)
     args = GdrHeadNormArgs()
     args.abi_version = ABI_VERSION
     args.tokens, args.head_dim, args.q_heads, args.k_heads = x.shape[0], head_dim, q_heads, k_heads
@@ -577,8 +585,9 @@ def head_norm(x, q_heads, k_heads, head_dim, q_weight, k_weight, eps) -> None:
 def swiglu(gate_up, out) -> None:
     """Enqueue gdr_swiglu_fwd on torch's current stream: out = silu(gate) * up for the first and second I columns of
     gate_up [T, >= 2 I], out [T, I] contiguous, both bf16."""
-    _expect("swiglu", "gate_up", gate_up, torch.bfloat16, out.device, (out.shape[0], 2 * out.shape[-1]), wider=True)
-    _expect("swiglu", "out", out, torch.bfloat16, out.device, (out.shape[0], out.shape[-1]))
+    _expect("swiglu", "out", out, torch.bfloat16, (out.shape[0], out.shape[-1]))
+    _expect("swiglu", "gate_up", gate_up, torch.bfloat16, (out.shape[0], 2 * out.shape[1]), wider=True)
+    _expect_one_gpu("swiglu", gate_up, out)
     args = GdrSwigluArgs()
     args.abi_version = ABI_VERSION
     args.rows, args.dim = out.shape

@@ -132,3 +132,24 @@ def test_mlp_weights_of_other_sizes():
     full, _ = model.forward(hidden, cu)
     # silu(gate) rounded to bf16 in between, or not: 2^-8 of the MLP's share of the stream
     assert (one - full).norm() <= 2.0 ** -8 * (full - hidden).norm()
+
+
+def test_attention_weights_of_other_sizes():
+    """q, k and v weights split otherwise than the configuration says, and norm weights of another length, are refused; a
+    norm weight of one value broadcasts, as in PyTorch."""
+    model, hidden, cu = _small_stack()
+    w = model.layers[1]
+    kept = dict(w)
+    bad = [{"wq": kept["wq"][:64], "wk": torch.cat([kept["wk"], kept["wk"]])}, {"wv": kept["wv"][:32]},
+           {"wk": torch.cat([kept["wk"], kept["wk"]])}, {"q_norm": torch.ones(32, device="cuda")},
+           {"k_norm": torch.ones(64)}]
+    for change in bad:
+        w.update(kept, **change)
+        with pytest.raises(RuntimeError):
+            model.forward(hidden, cu)
+    w.update(kept, q_norm=torch.full((64,), 1.5, device="cuda"))
+    full, _ = model.forward(hidden, cu)
+    w["q_norm"] = torch.full((1,), 1.5, device="cuda")
+    one, _ = model.forward(hidden, cu)
+    # one rounding of q (2^-8 of a score's scale), none elsewhere: 2^-7 of what the layer adds is ample
+    assert (one - full).norm() <= 2.0 ** -7 * (full - hidden).norm()

@@ -435,3 +435,14 @@ def test_swiglu_wrapper_checks_shapes_before_any_pointer():
         lib.swiglu(torch.empty(192, 5, dtype=torch.bfloat16).t(), out)
     with pytest.raises(ValueError, match="GPU"):
         lib.swiglu(torch.empty(5, 192, dtype=torch.bfloat16), out)
+
+
+def test_head_norm_wrapper_checks_shapes_before_any_pointer():
+    x, w = torch.empty(5, 3 * 64, dtype=torch.bfloat16), torch.ones(64)
+    for q, k, name in ((torch.ones(1), w, "q_weight"), (w, torch.ones(32), "k_weight"), (w.double(), w, "q_weight")):
+        with pytest.raises(ValueError, match=name):
+            lib.head_norm(x, 2, 1, 64, q, k, 1e-6)
+    with pytest.raises(ValueError, match="head_norm: x"):
+        lib.head_norm(x, 3, 1, 64, w, w, 1e-6)
+    with pytest.raises(ValueError, match="GPU"):
+        lib.head_norm(x, 2, 1, 64, w, w, 1e-6)
