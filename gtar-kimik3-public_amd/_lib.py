@@ -548,8 +548,16 @@ def _expect_one_gpu(op, *tensors) -> None:
 def add_norm(residual, add, weight, eps, total, out) -> None:
     """Enqueue gdr_add_norm_fwd on torch's current stream: total = residual + add, out = rmsnorm(total) * weight over
     contiguous [rows, dim] tensors; add, total and out may be None."""
-    if weight is not None and weight.numel() != residual.shape[-1]:
-        raise ValueError(f"add_norm: weight must have {residual.shape[-1]} values, got {tuple(weight.shape)}")
+    if residual.dtype not in (torch.float32, torch.bfloat16):
+        raise ValueError(f"add_norm: residual must be float32 or bfloat16, got {residual.dtype}")
+    shape = (residual.shape[0], residual.shape[-1])
+    for name, t, dtype in (("residual", residual, residual.dtype), ("add", add, torch.bfloat16),
+                           ("sum", total, torch.float32), ("out", out, torch.bfloat16)):
+        if t is not None:
+            _expect("add_norm", name, t, dtype, shape)
+    if weight is not None:
+        _expect("add_norm", "weight", weight, torch.float32, shape[1:])
+    _expect_one_gpu("add_norm", residual, add, weight, total, out)
     args = GdrAddNormArgs()
     args.abi_version = ABI_VERSION
     args.rows, args.dim = residual.shape

@@ -153,3 +153,25 @@ def test_attention_weights_of_other_sizes():
     one, _ = model.forward(hidden, cu)
     # one rounding of q (2^-8 of a score's scale), none elsewhere: 2^-7 of what the layer adds is ample
     assert (one - full).norm() <= 2.0 ** -7 * (full - hidden).norm()
+
+
+def test_residual_weights_of_other_sizes():
+    """Projections back to the stream of another width and block norm weights of another length or on the CPU are refused;
+    a norm weight of one value and a down projection of one row broadcast, as in PyTorch."""
+    model, hidden, cu = _small_stack()
+    w = model.layers[1]
+    kept = dict(w)
+    for change in ({"wo": kept["wo"][:64]}, {"down": kept["down"][:64]}, {"in_norm": torch.ones(64, device="cuda")},
+                   {"post_norm": torch.ones(128)}):
+        w.update(kept, **change)
+        with pytest.raises(RuntimeError):
+            model.forward(hidden, cu)
+    for name, one, full in (("in_norm", torch.full((1,), 1.5, device="cuda"), torch.full((128,), 1.5, device="cuda")),
+                            ("post_norm", torch.full((1,), 1.5, device="cuda"), torch.full((128,), 1.5, device="cuda")),
+                            ("down", kept["down"][:1].clone(), kept["down"][:1].expand(128, 96).contiguous())):
+        w.update(kept, **{name: full})
+        want, _ = model.forward(hidden, cu)
+        w[name] = one
+        got, _ = model.forward(hidden, cu)
+        # another order of the row's sum moves some bf16 operands by one rounding (2^-8)
+        assert (got - want).norm() <= 2.0 ** -7 * (want - hidden).norm(), name

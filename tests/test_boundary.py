@@ -446,3 +446,18 @@ def test_head_norm_wrapper_checks_shapes_before_any_pointer():
         lib.head_norm(x, 3, 1, 64, w, w, 1e-6)
     with pytest.raises(ValueError, match="GPU"):
         lib.head_norm(x, 2, 1, 64, w, w, 1e-6)
+
+
+def test_add_norm_wrapper_checks_shapes_before_any_pointer():
+    h, y, w = torch.empty(5, 64), torch.empty(5, 64, dtype=torch.bfloat16), torch.ones(64)
+    total, x = torch.empty(5, 64), torch.empty(5, 64, dtype=torch.bfloat16)
+    for args, name in (((h, y[:, :1], w, 1e-6, total, x), "add"), ((h, y[:4], w, 1e-6, total, x), "add"),
+                       ((h, y, w[:32], 1e-6, total, x), "weight"), ((h, y, w, 1e-6, total[:, :32], x), "sum"),
+                       ((h, y, w, 1e-6, total, x[:4]), "out"), ((h.half(), y, w, 1e-6, total, x), "residual"),
+                       ((h, y.float(), w, 1e-6, total, x), "add")):
+        with pytest.raises(ValueError, match=f"add_norm: {name} must be"):
+            lib.add_norm(*args)
+    with pytest.raises(ValueError, match="contiguous"):
+        lib.add_norm(h, y, torch.ones(64, 2)[:, 0], 1e-6, total, x)
+    with pytest.raises(ValueError, match="GPU"):
+        lib.add_norm(h, y, w, 1e-6, total, x)
