@@ -502,6 +502,12 @@ def short_conv(x, out, weight, state_in, state_out, cu_seqlens, silu, device) ->
 def norm_gate(x, gate, weight, out, eps, device) -> None:
     """Enqueue gdr_norm_gate_fwd (gdr_norm_gate_rounded_fwd for an fp32 weight and a 16-bit `out`) on torch's current
     stream; x, gate, out are [B, T, H, V] views."""
+    if gate.shape != x.shape or out.shape != x.shape or tuple(weight.shape) != x.shape[3:]:
+        raise ValueError(f"norm_gate: gate and out must be {list(x.shape)} and weight {list(x.shape[3:])}, got "
+                         f"{list(gate.shape)}, {list(out.shape)} and {list(weight.shape)}")
+    if not weight.is_contiguous():
+        raise ValueError("norm_gate: weight must be contiguous")
+    _expect_one_gpu("norm_gate", x, gate, weight, out)
     args = GdrNormGateArgs()
     args.abi_version = ABI_VERSION
     args.batch, args.seq_len, args.heads, args.value_dim = x.shape

@@ -21,6 +21,11 @@ def output_norm_gate(x: torch.Tensor, gate: torch.Tensor, weight: torch.Tensor, 
     """weight * rmsnorm(x) * silu(gate) for x, gate [B, T, H, V] (x may be the op's [B, H, T, V] output transposed),
     weight [V].  Returns [B, T, H, V], float32 when the weight is float32 (PyTorch's type promotion), else x's
     dtype."""
+    return norm_gate(x, gate, weight, eps, rounded=False)
+
+
+def norm_gate(x, gate, weight, eps, rounded: bool) -> torch.Tensor:
+    """output_norm_gate; with `rounded`, a float32 weight's result in x's dtype, rounded once more on the way out."""
     name = "output_norm_gate"
     if torch.is_grad_enabled() and any(t.requires_grad for t in (x, gate, weight)):
         raise NotImplementedError(f"{name}: forward only; run under torch.no_grad()")
@@ -40,7 +45,7 @@ def output_norm_gate(x: torch.Tensor, gate: torch.Tensor, weight: torch.Tensor, 
         if t.stride(-1) != 1 or t.data_ptr() % 16 or any((s * t.element_size()) % 16 for s in t.stride()[:3]):
             t = t.contiguous()
         views.append(t)
-    out_dtype = torch.float32 if weight.dtype == torch.float32 else x.dtype
+    out_dtype = torch.float32 if weight.dtype == torch.float32 and not rounded else x.dtype
     out = torch.empty(x.shape, device=x.device, dtype=out_dtype)
     _lib.norm_gate(views[0], views[1], weight, out, eps, x.device)
     return out

@@ -175,3 +175,18 @@ def test_residual_weights_of_other_sizes():
         got, _ = model.forward(hidden, cu)
         # another order of the row's sum moves some bf16 operands by one rounding (2^-8)
         assert (got - want).norm() <= 2.0 ** -7 * (want - hidden).norm(), name
+
+
+def test_kda_norm_weights_of_other_sizes():
+    """The KDA mixer's output norm takes one weight per value channel, on the stack's GPU; a 16-bit one is used as it is."""
+    model, hidden, cu = _small_stack()
+    w = model.layers[0]
+    for norm in (torch.ones(32, device="cuda"), torch.ones(1, device="cuda"), torch.ones(64)):
+        w["norm"] = norm
+        with pytest.raises(ValueError, match="output_norm_gate"):
+            model.forward(hidden, cu)
+    w["norm"] = torch.full((64,), 1.5, device="cuda")
+    want, _ = model.forward(hidden, cu)
+    w["norm"] = w["norm"].bfloat16()
+    got, _ = model.forward(hidden, cu)
+    assert (got - want).norm() <= 2.0 ** -7 * (want - hidden).norm()  # one more bf16 rounding (2^-8) of each product

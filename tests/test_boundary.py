@@ -461,3 +461,15 @@ def test_add_norm_wrapper_checks_shapes_before_any_pointer():
         lib.add_norm(h, y, torch.ones(64, 2)[:, 0], 1e-6, total, x)
     with pytest.raises(ValueError, match="GPU"):
         lib.add_norm(h, y, w, 1e-6, total, x)
+
+
+def test_norm_gate_wrapper_checks_shapes_before_any_pointer():
+    x = torch.empty(1, 4, 2, 64, dtype=torch.bfloat16)
+    for gate, w, out in ((x, torch.ones(32), x), (x, torch.ones(1), x), (x[:, :3], torch.ones(64), x),
+                         (x, torch.ones(64), x[..., :32])):
+        with pytest.raises(ValueError, match="norm_gate: gate and out must be"):
+            lib.norm_gate(x, gate, w, out, 1e-6, x.device)
+    with pytest.raises(ValueError, match="contiguous"):
+        lib.norm_gate(x, x, torch.ones(64, 2)[:, 0], x, 1e-6, x.device)
+    with pytest.raises(ValueError, match="GPU"):
+        lib.norm_gate(x, x, torch.ones(64), x, 1e-6, x.device)
