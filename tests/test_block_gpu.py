@@ -190,3 +190,32 @@ def test_kda_norm_weights_of_other_sizes():
     w["norm"] = w["norm"].bfloat16()
     got, _ = model.forward(hidden, cu)
     assert (got - want).norm() <= 2.0 ** -7 * (want - hidden).norm()  # one more bf16 rounding (2^-8) of each product
+
+
+def test_f16_autocast_keeps_f16_operands():
+    """Under autocast to f16 the projections' results, the attention, the MLP's product and the addends keep f16's 11 bits:
+    the error of an attention layer's update against fp64 blocks is an eighth of bf16's by the operand types alone, and
+    held to half of it.  The projections' inputs are the bf16 norms either way, so the reference takes those."""
+    cfg = stack.StackConfig(hidden_size=256, intermediate_size=384, num_layers=1, num_attention_heads=4,
+                            num_key_value_heads=2, head_dim=64, attention_interval=1)
+    layers = stack.init_weights(cfg, seed=3)
+    w = {k: (t.double().cuda() if torch.is_tensor(t) else t) for k, t in layers[0].items()}
+    cu, hidden = torch.tensor([0, 70], dtype=torch.int32, device="cuda"), _rand(1, 70, 256, seed=13)
+    rms = lambda t, weight: t * torch.rsqrt(t.pow(2).mean(-1, keepdim=True) + cfg.rms_norm_eps) * weight
+    h = hidden[0].double()
+    x = rms(h, w["in_norm"]).bfloat16().double()
+    q, k, v = ((x @ w[n].t()).view(70, -1, 64).transpose(0, 1) for n in ("wq", "wk", "wv"))
+    k, v = (t.repeat_interleave(2, 0) for t in (rms(k, w["k_norm"]), v))
+    s = (rms(q, w["q_norm"]) @ k.transpose(1, 2).contiguous()) / 8
+    s = s.masked_fill(torch.ones(70, 70, dtype=torch.bool, device="cuda").triu(1), float("-inf")).softmax(-1)
+    h = h + (s @ v).transpose(0, 1).reshape(70, -1) @ w["wo"].t()
+    x = rms(h, w["post_norm"]).bfloat16().double()
+    ref = h + (F.silu(x @ w["gate"].t()) * (x @ w["up"].t())) @ w["down"].t()
+    model = stack.HybridStack(cfg, layers)
+    err = {}
+    for dtype in (torch.float16, torch.bfloat16):
+        with torch.autocast("cuda", dtype):
+            out, _ = model.forward(hidden, cu)
+        err[dtype] = ((out[0].double() - ref).norm() / (ref - hidden[0].double()).norm()).item()
+    print(f"error of the update: f16 {err[torch.float16]:.2e}, bf16 {err[torch.bfloat16]:.2e}")
+    assert err[torch.float16] <= 0.5 * err[torch.bfloat16]
