@@ -219,3 +219,18 @@ def test_f16_autocast_keeps_f16_operands():
         err[dtype] = ((out[0].double() - ref).norm() / (ref - hidden[0].double()).norm()).item()
     print(f"error of the update: f16 {err[torch.float16]:.2e}, bf16 {err[torch.bfloat16]:.2e}")
     assert err[torch.float16] <= 0.5 * err[torch.bfloat16]
+
+
+def test_weights_on_the_device_stay_the_callers():
+    """A stack of tensors that are on the device already keeps them: no second copy, and updates in place reach it."""
+    moved, hidden, cu = _small_stack()
+    given = [{k: (t.clone() if torch.is_tensor(t) else t) for k, t in w.items() if k not in ("wqkv", "gate_up")}
+             for w in moved.layers]
+    kept = stack.HybridStack(moved.cfg, given)
+    for w, g in zip(kept.layers, given):
+        assert all(w[k] is g[k] for k in g)
+    assert torch.equal(kept.forward(hidden, cu)[0], moved.forward(hidden, cu)[0])
+    for name in ("wq", "wk", "wv", "gate", "up"):
+        for w in (given[1], moved.layers[1]):
+            w[name].mul_(0.5)
+    assert torch.equal(kept.forward(hidden, cu)[0], moved.forward(hidden, cu)[0])
