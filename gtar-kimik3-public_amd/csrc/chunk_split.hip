@@ -541,7 +541,10 @@ __global__ __launch_bounds__(256, ((__is_same(T, _Float16) && (VARIANT == GDR_KD
     }
   }
   if constexpr (kGate == 1) {
-    const float g = x.gp[tc * x.g_st];
+    // A gate below kReset is a reset: e^g is 0 in fp32 there (-inf included), and held at kReset it leaves the prefix sums
+    // of the tokens around it their precision, which every decay between two tokens is the difference of (a NaN stays).
+    constexpr float kReset = -104.f;
+    const float raw = x.gp[tc * x.g_st], g = raw < kReset ? kReset : raw;
 #pragma unroll
     for (int kk = 0; kk < KS; ++kk)
 #pragma unroll
@@ -642,10 +645,12 @@ __global__ __launch_bounds__(256, ((__is_same(T, _Float16) && (VARIANT == GDR_KD
   // f16 operands: the diagonal strip tile runs on bf16 operands formed here in fp32 (see step 4)
   constexpr bool kWideDiag = kGate == 2 && __is_same(T, _Float16);
   // A scalar gate: the diagonal tile is the plain q k^T (k k^T) product times e^{B_t - B_s} per element, in fp32, from
-  // this lane's own rows (exact for any gate, so there is no hot case).  Its products run here, before the rows are
-  // scaled, so that nothing is held for them: the f16 build, which formed bf16 operands for this tile, fits three
-  // workgroups per CU without those, and its error falls (GDN, B = 2, T = 8,111, f16: 269 -> 251 us per call with the
-  // hinted loads, output error 2.4e-3 -> 4.7e-4; bf16 4.7e-3 -> 3.7e-3 at an unchanged time).
+  // this lane's own rows.  The factor needs no hot case; as the difference of two fp32 prefix sums its relative error is
+  // about half an ulp of the larger one: 4e-6 among ordinary gates, 1e-5 after a reset in the block (held at kReset: |B| <
+  // 256), 2e-4 were every token one.  The products run here, before the rows are scaled, so that nothing is held for
+  // them: the f16 build, which formed bf16 operands for this tile, fits three workgroups per CU without those, and its
+  // error falls (GDN, B = 2, T = 8,111, f16: 269 -> 251 us per call with the hinted loads; output error against fp64, 2-norm
+  // over 2-norm, 2.4e-3 -> 4.7e-4, final state 3.2e-4 -> 3.1e-4; bf16 4.6e-3 -> 3.7e-3 at an unchanged time).
   constexpr bool kScalarDiag = kGate == 1;
   floatx4 diag_s = {0.f, 0.f, 0.f, 0.f}, diag_p = {0.f, 0.f, 0.f, 0.f};
   bf16x8 dq[kWideDiag ? KS : 1], dk[kWideDiag ? KS : 1], dkey[kWideDiag ? KS : 1];

@@ -43,3 +43,15 @@ def test_decay_ranges(dtype, gate_scale, T, K):
 def test_hinted_loads(dtype):
     inp = workloads.make_inputs("gdn", 4, 4000, 16, 128, 128, seed=3, dtype=DTYPES[dtype], state_std=0.02, device="cuda")
     _check(inp, dtype, keep=slice(3, 4))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("reset", [-60.0, -1e3, -1e5, -1e7, -1e9, torch.finfo(torch.float32).min, -float("inf")])
+@pytest.mark.parametrize("T", [63, 333])
+def test_resets_among_ordinary_gates(dtype, reset, T):
+    """A gate that empties the state, at one token in eight, among ordinary ones: the decays between the tokens on either
+    side of it are differences of prefix sums that contain it."""
+    inp = workloads.make_inputs("gdn", 2, T, 3, 128, 64, seed=T, dtype=DTYPES[dtype], state_std=0.5, device="cuda")
+    at = torch.rand(inp.gate.shape, generator=torch.Generator().manual_seed(1)) < 0.125
+    inp.gate = inp.gate.masked_fill(at.cuda(), reset)
+    _check(inp, dtype)
