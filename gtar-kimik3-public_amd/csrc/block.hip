@@ -16,6 +16,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kRowsPerBlock = kThreads / kWave;
+static_assert(kRowsPerBlock == kAddNormRows && kThreads / 16 == kHeadNormRows, "row limits of the entry points");
 
 using bf16x8 = __bf16 __attribute__((ext_vector_type(8)));
 using f32x4 = float __attribute__((ext_vector_type(4)));
@@ -203,9 +204,7 @@ hipError_t launch_head_norm(const gdr_head_norm_args& a, hipStream_t stream) {
 
 hipError_t launch_swiglu(const gdr_swiglu_args& a, hipStream_t stream) {
   if (a.rows == 0) return hipSuccess;
-  const uintptr_t bits = reinterpret_cast<uintptr_t>(a.gate) | reinterpret_cast<uintptr_t>(a.up) |
-                         reinterpret_cast<uintptr_t>(a.out);
-  const bool wide = a.dim % 8 == 0 && a.stride % 8 == 0 && bits % 16 == 0;
+  const bool wide = swiglu_wide(a);
   const int64_t n = a.rows * (wide ? a.dim / 8 : a.dim);
   const dim3 grid(unsigned((n + kThreads - 1) / kThreads));
   if (wide) hipLaunchKernelGGL((swiglu_kernel<8>), grid, dim3(kThreads), 0, stream, a);

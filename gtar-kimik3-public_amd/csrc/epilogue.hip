@@ -18,6 +18,7 @@ namespace {
 
 constexpr float kLog2eF = 1.4426950408889634f;
 constexpr int kIter = 4;  // rows in flight per thread
+static_assert(16 * kIter == kNormGateRows, "row limit of the entry point");
 
 template <typename T>
 __device__ __forceinline__ float to_f(T v) { return static_cast<float>(v); }
@@ -50,7 +51,7 @@ __global__ __launch_bounds__(256) void norm_gate_kernel(const gdr_norm_gate_args
   int64_t xo[kIter], go[kIter], oo[kIter];
 #pragma unroll
   for (int it = 0; it < kIter; ++it) {  // row row0 + 16 it (clamped: rows past the end are computed, not stored)
-    const uint32_t row = uint32_t(min(row0 + 16 * it, rows - 1));  // rows < 2^31 (checked on the host)
+    const uint32_t row = uint32_t(min(row0 + 16 * it, rows - 1));  // rows < 2^30 (checked on the host)
     const uint32_t h = row % uint32_t(a.heads), bt = row / uint32_t(a.heads);
     const uint32_t t = bt % uint32_t(a.seq_len), b = bt / uint32_t(a.seq_len);
     xo[it] = int64_t(b) * a.x.stride_b + int64_t(t) * a.x.stride_t + int64_t(h) * a.x.stride_h + c0;

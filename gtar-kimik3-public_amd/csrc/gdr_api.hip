@@ -289,8 +289,8 @@ int norm_gate(const gdr_norm_gate_args* a, bool rounded, hipStream_t stream) {
     return fail(GDR_ERR_INVALID, "bad sizes B=%d T=%d H=%d", a->batch, a->seq_len, a->heads);
   if (a->value_dim < 64 || a->value_dim > 256 || a->value_dim % 64)
     return fail(GDR_ERR_UNSUPPORTED, "value dim %d not supported (64, 128, 192 or 256)", a->value_dim);
-  if (int64_t(a->batch) * a->seq_len * a->heads >= (int64_t(1) << 31))
-    return fail(GDR_ERR_UNSUPPORTED, "B * T * H must be below 2^31");
+  if (int64_t(a->batch) * a->seq_len > gdr::kMaxBlocks * gdr::kNormGateRows / a->heads)
+    return fail(GDR_ERR_UNSUPPORTED, "B * T * H must be at most %lld", (long long)(gdr::kMaxBlocks * gdr::kNormGateRows));
   if (!(a->eps >= 0.f)) return fail(GDR_ERR_INVALID, "eps must be >= 0");
   int rc;
   if ((rc = check_view(a->x, "x", true, false)) || (rc = check_view(a->gate, "gate", true, false)) ||
@@ -515,8 +515,10 @@ int gdr_add_norm_fwd(const gdr_add_norm_args* a, hipStream_t stream) {
   if (!a) return fail(GDR_ERR_INVALID, "args is NULL");
   if (a->abi_version != GDR_ABI_VERSION)
     return fail(GDR_ERR_INVALID, "abi_version %d, library implements %d", a->abi_version, GDR_ABI_VERSION);
-  if (a->dim < 1 || a->rows < 0 || a->rows >= (int64_t(1) << 31))
+  if (a->dim < 1 || a->rows < 0)
     return fail(GDR_ERR_INVALID, "bad sizes rows=%lld dim=%d", (long long)a->rows, a->dim);
+  if (a->rows > gdr::kMaxBlocks * gdr::kAddNormRows)
+    return fail(GDR_ERR_UNSUPPORTED, "rows must be at most %lld", (long long)(gdr::kMaxBlocks * gdr::kAddNormRows));
   if (a->residual_dtype != GDR_F32 && a->residual_dtype != GDR_BF16)
     return fail(GDR_ERR_UNSUPPORTED, "residual must be f32 or bf16 (got dtype code %d)", a->residual_dtype);
   if (a->rows && !a->residual) return fail(GDR_ERR_INVALID, "residual: null pointer");
@@ -534,11 +536,13 @@ int gdr_head_norm_fwd(const gdr_head_norm_args* a, hipStream_t stream) {
     return fail(GDR_ERR_INVALID, "abi_version %d, library implements %d", a->abi_version, GDR_ABI_VERSION);
   if (a->head_dim != 64 && a->head_dim != 128)
     return fail(GDR_ERR_UNSUPPORTED, "head dim %d not supported (64 or 128)", a->head_dim);
-  if (a->q_heads < 0 || a->k_heads < 0 || a->q_heads + a->k_heads < 1 || a->tokens < 0 ||
-      a->tokens * (a->q_heads + a->k_heads) >= (int64_t(1) << 31) ||
-      a->stride_t < int64_t(a->q_heads + a->k_heads) * a->head_dim)
+  const int64_t heads = int64_t(a->q_heads) + a->k_heads;
+  if (a->q_heads < 0 || a->k_heads < 0 || heads < 1 || a->tokens < 0 || a->stride_t < heads * a->head_dim)
     return fail(GDR_ERR_INVALID, "bad sizes tokens=%lld heads=%d + %d stride=%lld", (long long)a->tokens, a->q_heads,
                 a->k_heads, (long long)a->stride_t);
+  if (a->tokens > gdr::kMaxBlocks * gdr::kHeadNormRows / heads)
+    return fail(GDR_ERR_UNSUPPORTED, "tokens * heads must be at most %lld",
+                (long long)(gdr::kMaxBlocks * gdr::kHeadNormRows));
   if (a->tokens && (!a->x || !a->q_weight || !a->k_weight)) return fail(GDR_ERR_INVALID, "null pointer");
   if (reinterpret_cast<uintptr_t>(a->x) % 16 || a->stride_t % 8)
     return fail(GDR_ERR_INVALID, "x: rows must be 16-byte aligned");
@@ -553,9 +557,12 @@ int gdr_swiglu_fwd(const gdr_swiglu_args* a, hipStream_t stream) {
   if (!a) return fail(GDR_ERR_INVALID, "args is NULL");
   if (a->abi_version != GDR_ABI_VERSION)
     return fail(GDR_ERR_INVALID, "abi_version %d, library implements %d", a->abi_version, GDR_ABI_VERSION);
-  if (a->dim < 1 || a->rows < 0 || a->stride < a->dim || a->rows * a->dim >= (int64_t(1) << 39))
+  if (a->dim < 1 || a->rows < 0 || a->stride < a->dim)
     return fail(GDR_ERR_INVALID, "bad sizes rows=%lld dim=%d stride=%lld", (long long)a->rows, a->dim,
                 (long long)a->stride);
+  const int64_t most = gdr::kMaxBlocks * 256 * (gdr::swiglu_wide(*a) ? 8 : 1);  // a thread takes 8 values, or one
+  if (a->rows > most / a->dim)
+    return fail(GDR_ERR_UNSUPPORTED, "rows * dim must be at most %lld (with these alignments)", (long long)most);
   if (a->rows && (!a->gate || !a->up || !a->out)) return fail(GDR_ERR_INVALID, "null pointer");
   hipError_t e = gdr::launch_swiglu(*a, stream);
   if (e != hipSuccess) return fail(GDR_ERR_HIP, "swiglu launch failed: %s", hipGetErrorString(e));

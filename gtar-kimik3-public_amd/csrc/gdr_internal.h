@@ -46,6 +46,17 @@ hipError_t launch_short_conv(const gdr_conv_args& a, hipStream_t stream);
 // The layer's output epilogue (RMSNorm x SiLU gate); arguments validated.
 hipError_t launch_norm_gate(const gdr_norm_gate_args& a, hipStream_t stream);
 
+// Most 256-thread workgroups of a launch: a grid dimension holds fewer than 2^32 threads.
+constexpr int64_t kMaxBlocks = (int64_t(1) << 24) - 1;
+
+// Rows per workgroup of the kernels below, and whether a SwiGLU call moves 8 values per thread (16-byte rows) or 1.
+constexpr int kNormGateRows = 64, kAddNormRows = 4, kHeadNormRows = 16;
+inline bool swiglu_wide(const gdr_swiglu_args& a) {
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(a.gate) | reinterpret_cast<uintptr_t>(a.up) |
+                         reinterpret_cast<uintptr_t>(a.out);
+  return a.dim % 8 == 0 && a.stride % 8 == 0 && bits % 16 == 0;
+}
+
 // The stack's residual adds and norms, head norms and SwiGLU product; arguments validated.
 hipError_t launch_add_norm(const gdr_add_norm_args& a, hipStream_t stream);
 hipError_t launch_head_norm(const gdr_head_norm_args& a, hipStream_t stream);

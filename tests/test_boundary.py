@@ -473,3 +473,28 @@ def test_norm_gate_wrapper_checks_shapes_before_any_pointer():
         lib.norm_gate(x, x, torch.ones(64, 2)[:, 0], x, 1e-6, x.device)
     with pytest.raises(ValueError, match="GPU"):
         lib.norm_gate(x, x, torch.ones(64), x, 1e-6, x.device)
+
+
+def test_block_entry_points_refuse_more_than_a_launch_holds():
+    """At most 2^24 - 1 workgroups of 256 threads: the largest admitted size gets as far as the pointer check, one more (and
+    sizes whose products leave 64 bits) is refused as a size."""
+    so = lib.load_library()
+    blocks = 2 ** 24 - 1
+
+    def refused(entry, args, field, most):
+        for n, rc in ((most, -1), (most + 1, -2), (2 ** 63 - 1, -2)):
+            if n < 2 ** (8 * ctypes.sizeof(dict(type(args)._fields_)[field]) - 1):
+                setattr(args, field, n)
+                assert getattr(so, entry)(ctypes.byref(args), None) == rc, (entry, n)
+                assert (b"null pointer" if rc == -1 else b"must be at most") in so.gdr_last_error()
+
+    a = lib.GdrAddNormArgs(abi_version=lib.ABI_VERSION, dim=64, residual_dtype=lib.F32)
+    refused("gdr_add_norm_fwd", a, "rows", 4 * blocks)
+    h = lib.GdrHeadNormArgs(abi_version=lib.ABI_VERSION, head_dim=64, q_heads=4, k_heads=2, stride_t=384)
+    refused("gdr_head_norm_fwd", h, "tokens", 16 * blocks // 6)
+    for dim, most in ((96, 8 * 256 * blocks // 96), (97, 256 * blocks // 97)):
+        s = lib.GdrSwigluArgs(abi_version=lib.ABI_VERSION, dim=dim, stride=2 * dim)
+        refused("gdr_swiglu_fwd", s, "rows", most)
+    n = lib.GdrNormGateArgs(abi_version=lib.ABI_VERSION, batch=1, heads=2, value_dim=64)
+    for entry in ("gdr_norm_gate_fwd", "gdr_norm_gate_rounded_fwd"):
+        refused(entry, n, "seq_len", 32 * blocks)
