@@ -21,6 +21,21 @@ def _writable_in_place(state: torch.Tensor, dtype: torch.dtype) -> bool:
         not (state.requires_grad and torch.is_grad_enabled())
 
 
+def _span(t: torch.Tensor):
+    """The addresses [first, end) that t's elements lie between (strides are not negative)."""
+    first = t.data_ptr()
+    if t.numel() == 0:
+        return first, first
+    return first, first + t.element_size() * (1 + sum((n - 1) * s for n, s in zip(t.shape, t.stride())))
+
+
+def _apart(written, read) -> bool:
+    """Whether no tensor that a kernel writes shares memory with another one or with one that it reads (None: absent)."""
+    spans = sorted(map(_span, written))
+    return all(a[1] <= b[0] for a, b in zip(spans, spans[1:])) and \
+        all(a[1] <= b[0] or b[1] <= a[0] for a in spans for b in (_span(t) for t in read if t is not None))
+
+
 def short_convolution(
     hidden_states: torch.Tensor,
     weight: torch.Tensor,
@@ -59,10 +74,10 @@ def short_convolution(
     out = torch.empty(x.shape, device=x.device, dtype=x.dtype)
     # The kernel writes the new state of every sequence that has tokens; a sequence of length 0 (and every sequence
     # when T == 0, which launches nothing) keeps its state, as the reference's does.  It reads a copy of the old state
-    # and writes the caller's tensor where that has the kernel's type and layout, else a second copy.
+    # and writes the caller's tensor where that has the kernel's type and layout and holds no input, else a second copy.
     state_in = state_out = None
     if conv_state is not None:
-        in_place = _writable_in_place(conv_state, x.dtype)
+        in_place = _writable_in_place(conv_state, x.dtype) and _apart((conv_state,), (x, w, cu_seqlens))
         state_in = conv_state.clone() if in_place else conv_state.to(x.dtype).contiguous()
         state_out = conv_state if in_place else state_in.clone()
     _lib.short_conv(x, out, w, state_in, state_out, cu_seqlens, activation, x.device)

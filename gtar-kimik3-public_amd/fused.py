@@ -24,13 +24,7 @@ import torch
 
 from . import _lib
 from ._common import _VARIANT_NAMES, _as_row_aligned, _autocast, _check_devices, _wants_grad
-from .conv import _writable_in_place
-
-
-def _apart(tensors) -> bool:
-    """Whether no two contiguous tensors share memory."""
-    spans = sorted((t.data_ptr(), t.data_ptr() + t.numel() * t.element_size()) for t in tensors)
-    return all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
+from .conv import _apart, _writable_in_place
 
 
 def _aligned16(x: torch.Tensor) -> torch.Tensor:
@@ -119,9 +113,10 @@ def _fused(variant, query, key, value, gate_lowrank, gate_weight, gate_bias, a_l
                     raise ValueError(f"{name}: {nm} conv state must be [{n_states}, {ch}, {width - 1}], got "
                                      f"{tuple(st.shape)}")
             # The kernel reads a copy of the states (one launch for the three) and writes the caller's tensors where
-            # they have its type and layout and are three tensors, else a second copy; a sequence of length 0 keeps its
-            # state either way.
-            in_place = all(_writable_in_place(st, torch.bfloat16) for st in conv_states) and _apart(conv_states)
+            # they have its type and layout and share no memory with each other or an input, else a second copy; a
+            # sequence of length 0 keeps its state either way.
+            in_place = all(_writable_in_place(st, torch.bfloat16) for st in conv_states) and \
+                _apart(conv_states, (query, key, value, z, w, bias, a_log, beta, initial_state, cu_seqlens, *conv_w))
             flat = torch.cat([st.to(torch.bfloat16).reshape(-1) for st in conv_states])
             states_in = [x.view(st.shape) for x, st in zip(flat.split([st.numel() for st in conv_states]),
                                                            conv_states)]

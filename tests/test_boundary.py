@@ -498,3 +498,17 @@ def test_block_entry_points_refuse_more_than_a_launch_holds():
     n = lib.GdrNormGateArgs(abi_version=lib.ABI_VERSION, batch=1, heads=2, value_dim=64)
     for entry in ("gdr_norm_gate_fwd", "gdr_norm_gate_rounded_fwd"):
         refused(entry, n, "seq_len", 32 * blocks)
+
+
+def test_written_in_place_only_apart_from_what_is_read():
+    """Conv states are written by the kernel itself only where no input and no other state shares their memory."""
+    from importlib import import_module
+    apart = import_module("gtar-kimik3-public_amd.conv")._apart
+    buf = torch.zeros(4, 64)
+    rows = list(buf)
+    assert apart(rows[:3], (rows[3], None, buf[3:, ::2], torch.empty(0)))
+    assert apart((rows[0],), ()) and apart((buf[2:],), (buf[:2],))
+    assert not apart(rows[:3], (buf[2],)) and not apart((rows[0], buf[0, 8:16]), ())
+    assert not apart((buf[1],), (buf.t()[3:5],))  # a strided input around it
+    assert not apart((buf[0, 60:],), (buf.as_strided((2, 64), (62, 1)),))
+    assert not apart((buf[3, :1],), (buf.view(-1)[::64],)) and apart((buf[3, 1:],), (buf.view(-1)[::64],))

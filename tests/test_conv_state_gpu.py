@@ -117,3 +117,15 @@ def test_tokens_per_thread(dtype, total, W):
                 assert torch.equal(gdr.short_convolution(x[:, pos:end], w, one), out[:, pos:end]), (n, pos)
                 pos = end
             assert torch.equal(st[n:n + 1], one), n
+
+
+def test_short_convolution_state_inside_its_input():
+    """A state that is a row of the input (width 2) is replaced after every row is read."""
+    for row in (0, 40, 70):
+        x, w = _rand(1, 71, 64, seed=1), _rand(64, 1, 2, seed=2)
+        with torch.no_grad():
+            state = x[:, row:row + 1].clone().transpose(1, 2)
+            want = gdr.short_convolution(x.clone(), w, state)
+            inside = x[:, row:row + 1].transpose(1, 2)
+            got = gdr.short_convolution(x, w, inside)
+        assert torch.equal(want, got) and torch.equal(inside, state)
