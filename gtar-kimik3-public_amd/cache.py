@@ -23,10 +23,11 @@ class RecurrentCache:
     def __init__(self, batch_size: int, num_heads: int, head_dim: int, value_dim: int, inner_size: int,
                  conv_size: int, device, dtype):
         self.state = torch.zeros(batch_size, num_heads, head_dim, value_dim, device=device, dtype=torch.float32)
-        # One allocation, one fill; .data makes each state a tensor of its own (no view of the others to autograd, its
-        # own version counter), so writing one in place never touches the others' graph.
-        flat = torch.zeros(3, batch_size, inner_size, conv_size - 1, device=device, dtype=dtype)
-        self.conv_states = [state.data for state in flat]
+        # Three tensors with memory of their own, so that keeping or saving one keeps no other, and one fill for the three (of
+        # their bytes: any dtype; through .data, so that their version counters start at 0 as those of new tensors do).
+        self.conv_states = [torch.empty(batch_size, inner_size, conv_size - 1, device=device, dtype=dtype)
+                            for _ in range(3)]
+        torch._foreach_zero_([state.data.view(torch.uint8) for state in self.conv_states])
         self.seq_len = 0
         self._snapshot = None
 

@@ -144,6 +144,20 @@ def test_recurrent_cache_conv_states_are_independent_tensors():
     assert torch.count_nonzero(second) == torch.count_nonzero(third) == 0
 
 
+def test_recurrent_cache_conv_states_have_memory_of_their_own(tmp_path):
+    from safetensors.torch import load_file, save_file
+    for dtype in (torch.bfloat16, torch.float16, torch.float32, torch.float64):
+        cache = gdr.RecurrentCache(2, 2, 4, 4, 8, 4, "cpu", dtype)
+        for state in cache.conv_states:
+            assert state.untyped_storage().nbytes() == state.numel() * state.element_size()
+    save_file(dict(zip("qkv", cache.conv_states)), tmp_path / "tails.safetensors")  # refuses tensors that share memory
+    assert all(torch.equal(load_file(tmp_path / "tails.safetensors")[n], s) for n, s in zip("qkv", cache.conv_states))
+    with torch.inference_mode():
+        cache = gdr.RecurrentCache(2, 2, 4, 4, 8, 4, "cpu", torch.bfloat16)
+    assert all(torch.count_nonzero(state) == 0 for state in cache.conv_states)
+    assert [tuple(s.shape) for s in gdr.RecurrentCache(2, 2, 4, 4, 8, 1, "cpu", torch.bfloat16).conv_states] == [(2, 8, 0)] * 3
+
+
 def test_recurrent_cache_fork_rollback_restores_state():
     cache = gdr.RecurrentCache(2, 2, 4, 4, 8, 4, "cpu", torch.float32)
     cache.update(torch.randn(2, 2, 4, 4), 3)
