@@ -170,14 +170,22 @@ hipError_t launch_conv_tok(const gdr_conv_args& a, hipStream_t stream) {
 
 template <typename T>
 hipError_t launch_conv_typed(const gdr_conv_args& a, hipStream_t stream) {
-  // Tokens per thread by the call's size, in 16-byte pieces of 8 tokens: more of them share the halo rows, fewer leave
-  // more threads in flight (and shorter chains at a sequence's ends, which run token by token).  Measured, us at 8 / 4 /
-  // 2 tokens, bf16, W = 4: [1, 333, 2048] 10.2 / 7.4 / 5.5, [2, 3001, 2048] (192 K pieces) 17.3 / 14.9 / 13.9,
-  // [4, 4096, 1024] (262 K) 22.4 / 17.2 / 16.7, [4, 4096, 2048] (524 K) 40.3 / 37.2 / 43.4, [2, 8192, 4096] (1,049 K)
-  // 59.5 / 59.7 / 73.1; f32 [2, 3001, 2048] (384 K) 19.8 / 18.5 / 17.9, [4, 4096, 2048] (1,049 K) 53.8 / 56.6 / 65.7.
+  // Tokens per thread by the call's size, in 16-byte pieces of 8 tokens: more of them share the W - 1 halo rows, fewer
+  // leave more threads in flight (and shorter chains at a sequence's ends, which run token by token); so the wider the
+  // convolution, the sooner a thread takes more.  Measured, us at 8 / 4 / 2 tokens, bf16:
+  //   W = 2  [4, 4096, 1024] (256 K pieces) 16.1 / 12.7 / 12.7, [4, 4096, 2048] (512 K) 23.1 / 24.2 / 21.4
+  //   W = 4  [1, 333, 2048] (10 K) 8.3 / 5.4 / 4.0, [4, 4096, 1024] 17.8 / 14.1 / 14.8, [4, 4096, 2048] 23.9 / 24.1 / 25.3,
+  //          [2, 8192, 4096] (1,024 K) 42.4 / 42.6 / 49.7
+  //   W = 6  [2, 3001, 2048] (188 K) 15.6 / 16.2 / 16.0, [4, 4096, 1024] 17.3 / 15.8 / 17.7, [4, 4096, 1536] (384 K)
+  //          20.8 / 20.8 / 24.5
+  //   W = 8  [1, 2000, 2048] (62 K) 18.6 / 12.1 / 10.6, [4, 4096, 1024] 23.2 / 21.7 / 30.3, [4, 4096, 1536]
+  //          25.8 / 29.6 / 43.6; f32 [1, 2000, 2048] (125 K) 11.8 / 10.0 / 13.9, [2, 3001, 1024] (188 K) 14.5 / 16.0 / 19.7
   const int64_t pieces = int64_t(a.cu_seqlens ? 1 : a.batch) * a.seq_len * a.channels * int(sizeof(T)) / (8 * 16);
-  if (pieces < 288 * 1024) return launch_conv_tok<T, 2>(a, stream);
-  if (pieces < 768 * 1024) return launch_conv_tok<T, 4>(a, stream);
+  const int W = a.kernel_size;
+  const int two = W <= 3 ? 768 : W == 4 ? 288 : W <= 6 ? 224 : 80;  // below this many K pieces: 2 tokens
+  const int four = W <= 4 ? 768 : W <= 6 || sizeof(T) == 2 ? 320 : 160;
+  if (pieces < two * 1024) return launch_conv_tok<T, 2>(a, stream);
+  if (pieces < four * 1024) return launch_conv_tok<T, 4>(a, stream);
   return launch_conv_tok<T, 8>(a, stream);
 }
 

@@ -95,12 +95,13 @@ def test_fused_prefill_states_that_are_not_written_in_place():
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
-@pytest.mark.parametrize("total", [4_000, 6_500, 13_001], ids=["2 tokens", "4 tokens", "8 tokens"])
+@pytest.mark.parametrize("total", [4_000, 6_500, 13_001], ids=["250 K pieces", "406 K", "813 K"])
 @pytest.mark.parametrize("W", [2, 4, 8])
 def test_tokens_per_thread(dtype, total, W):
-    """A thread takes 2, 4 or 8 tokens by the size of the call (bf16 at 4,096 channels: 288 K and 768 K pieces are 4,608
-    and 12,288 tokens; half that in f32).  Packed sequences with lengths around all three tiles, and one long one that
-    sets the size, equal each sequence's own (2-token) call bit for bit, states included."""
+    """A thread takes 2, 4 or 8 tokens by the size of the call (in K pieces of 16 bytes and 8 tokens, bf16 and f32 alike
+    here) and the width: 2, 4 and 8 at W = 4, 2, 2 and 8 at W = 2, 4 (f32: 8), 8 and 8 at W = 8.  Packed sequences with
+    lengths around all three tiles, and one long one that sets the size, equal each sequence's own (2-token, at most 63 K
+    pieces) call bit for bit, states included."""
     C = 4096 if dtype == torch.bfloat16 else 2048
     short = [1, 7, 8, 9, 0, 3, 4, 5, 16, 15, 17, 2, 41]
     lengths = short + [total - sum(short)]
@@ -112,8 +113,8 @@ def test_tokens_per_thread(dtype, total, W):
         out = gdr.short_convolution(x, w, st, cu_seqlens=cu.cuda())
         for n, (a, b) in enumerate(zip(cu[:-1].tolist(), cu[1:].tolist())):
             pos, one = a, state[n:n + 1].clone()
-            while pos < b:  # the long sequence in pieces that stay below the 4-token size, its state carried
-                end = min(b, pos + 4_001)
+            while pos < b:  # the long sequence in parts that stay below every 4-token size, its state carried
+                end = min(b, pos + 1_001)
                 assert torch.equal(gdr.short_convolution(x[:, pos:end], w, one), out[:, pos:end]), (n, pos)
                 pos = end
             assert torch.equal(st[n:n + 1], one), n
