@@ -10,8 +10,9 @@
 //
 // Design: the state is streamed exactly once per call (one 128-bit load and one 128-bit store per float4),
 // so the kernel is HBM-bound at T = 1.  One workgroup owns a [K, VS] column slice of one (b, h) state: 512
-// threads for 128-column slices (large batches), 256 for 64-column slices (one token, middle-sized batches) and for
-// 32-column slices (small batches, so they still launch enough workgroups).  Thread (quad, rg) holds float4 column quad `quad` of rows rg, rg + RG, ... in
+// threads for 128-column slices (large batches), 256 for 64-column slices (few tokens, middle-sized batches) and for
+// 32-column slices (small batches, so they still launch enough workgroups).  Thread (quad, rg) holds float4 column quad
+// `quad` of rows rg, rg + RG, ... in
 // registers for the whole call; few rows per thread keep the register count low enough for 6+ waves per SIMD,
 // which together with non-temporal state loads keeps enough bytes in flight.  Both dk-reductions (k S and q S)
 // come out of one pass over the registers, are reduced across lanes with shuffles and across waves through LDS,
@@ -50,15 +51,16 @@ static hipError_t launch_family(const gdr_args& a, hipStream_t stream, RecMode m
   // Narrow slices give small calls enough workgroups; wide ones spend less of the vector ALU on cross-lane sums (a
   // thread sums 8 rows of 4 columns, at 32 columns 4) and less LDS traffic per token.  From 32,768 columns the wide
   // ones win (us per call, KDA, H = 16, K = V = 128, 32 / 64 / 128 columns; 8 tokens: B = 8 11.2 / 11.0 / 11.4, B = 16
-  // 16.9 / 14.1 / 13.6, B = 48 38.5 / 28.8 / 28.0, a commit and verify cycle 44.7 / 38.9 / 34.2); one token, bound by
-  // the state stream, runs best on 64 (B = 24 11.0 / 9.4 / 10.4, B = 48 20.4 / 18.7 / 21.5) until the rounds of
-  // workgroups are many (B = 256 84.5 / 81.0 / 81.6 on one buffer, on fresh ones 99.8 against 99.3 at 128).
+  // 16.9 / 14.1 / 13.6, B = 48 38.5 / 28.8 / 28.0, a commit and verify cycle 44.7 / 38.9 / 34.2); up to four tokens, bound
+  // by the state stream, run best on 64 (one token: B = 24 11.0 / 9.4 / 10.4, B = 48 20.4 / 18.7 / 21.5; three: B = 33
+  // 19.3 / 17.6 / 18.8, DeltaNet 17.4 / 17.1 / 18.1) until the rounds of workgroups are many (B = 256, one token 84.5 / 81.0
+  // / 81.6 on one buffer, on fresh ones 99.8 against 99.3 at 128).
   // 64 and 128 agree bit for bit, 32 does not, so the choice between them depends on the tokens and that of 32 on the
   // columns alone: a verify, its commit and a recurrent call on part of the block agree bit for bit.
   const int64_t columns = int64_t(a.cu_seqlens ? a.n_seqs : a.batch) * a.heads * a.value_dim;
   int vs = 32;
   if (columns >= 32768 && a.value_dim % 64 == 0)
-    vs = a.value_dim % 128 == 0 && (a.seq_len > 1 || mode != RecMode::kForward || columns >= 131072) ? 128 : 64;
+    vs = a.value_dim % 128 == 0 && (a.seq_len > 4 || mode != RecMode::kForward || columns >= 131072) ? 128 : 64;
   if (a.key_dim != 64 && a.key_dim != 128) return launch_recurrent_other_k(a, stream, vs, mode, x, dtype);
   return dtype == GDR_BF16 ? launch_recurrent_t<__bf16>(a, stream, vs, mode, x)
                            : launch_recurrent_t<float>(a, stream, vs, mode, x);

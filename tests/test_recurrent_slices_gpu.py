@@ -1,5 +1,5 @@
 """The recurrent family's slice widths on the GPU: 32 columns below 32,768 (sequence, head, column) triples, and from
-there 64 columns for one-token calls (up to 131,072) and 128 for the others (64 throughout when the value dim is no
+there 64 columns for calls of up to four tokens (up to 131,072) and 128 for the others (64 throughout when the value dim is no
 multiple of 128).
 A one-token call and the first token of a longer verify agree bit for bit whatever slices they ran on, and both are
 within fp32 rounding of the fp64 recurrence (1e-5, plus the one rounding of a bf16 output)."""
@@ -37,3 +37,17 @@ def test_slice_widths_agree(variant, shape):
     q, k, v, g, beta, h0 = oracle_args(inp)
     ref_o, ref_s = oracle.recurrence(variant, q, k, v, g, beta, None, h0)
     assert out_error(out, ref_o) <= 1e-5 + 2.0 ** -8 and state_error(final, ref_s) <= 1e-5
+
+
+@pytest.mark.parametrize("variant", oracle.VARIANTS)
+def test_calls_of_four_and_five_tokens_agree(variant):
+    """Four tokens run on 64-column slices, five and the verify of six on 128: the same prefix bit for bit."""
+    inp = workloads.make_inputs(variant, 17, 6, 16, 128, 128, seed=2, state_std=0.5, device="cuda", layer_layout=True)
+    with torch.no_grad():
+        out, _, block = verify_op(VARIANTS[variant], inp.query, inp.key, inp.value, inp.gate, inp.beta,
+                                  initial_state=inp.initial_state)
+        for n in (4, 5):
+            part = [None if x is None else x[:, :, :n] for x in (inp.query, inp.key, inp.value, inp.gate, inp.beta)]
+            got, state = RECURRENT_FNS[variant](*(x for x in part if x is not None), initial_state=inp.initial_state,
+                                                output_final_state=True)
+            assert torch.equal(got, out[:, :, :n]) and torch.equal(state, block.commit(n)), n
