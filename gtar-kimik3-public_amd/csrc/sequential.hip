@@ -274,17 +274,26 @@ hipError_t launch_t(const gdr_args& a, hipStream_t stream) {
 
 // The recurrent kernel keeps the calls it serves better (us per call, recurrent / here, fp32 KDA, V = 128):
 //   * few tokens: its state loads and stores are whole rows, where a wave here touches CW columns of every row.  From
-//     8 tokens on this kernel wins (B = 2, H = 16, K = 128, T = 8: 8.5 / 6.2), for key dims above 128 (more state per
-//     column) and more than 8,192 columns from about 64 (B = 8, H = 24, K = 256: T = 16 32.5 / 38.2, T = 200 308 / 259);
-//   * calls that fill the chip with its 128-column workgroups at K = 128, where both are bound by the vector ALU and q, k
-//     and e^g cost those fewer LDS reads (H = 16, 16 / 100 tokens: B = 24 28.7 / 26.6 and 130 / 115, B = 32 30.5 / 33.9
-//     and 132 / 145, B = 64 53.8 / 61.1 and 259 / 296); at K = 32 and 64 the wide split stays ahead (B = 64, K = 64: 16
-//     tokens 38.1 / 33.9, 100 tokens 186 / 161).
+//     8 tokens on this kernel wins (B = 2, H = 16, K = 128, T = 8: 8.5 / 6.2), at K = 256 from 16 (B = 4, H = 16: T = 12
+//     16.8 / 17.3, T = 16 20.5 / 17.5), for key dims above 128 (more state per column) and more than 8,192 columns from
+//     about 64 (B = 8, H = 24, K = 256: T = 16 32.5 / 38.2, T = 200 308 / 259);
+//   * calls that fill the chip with its workgroups: at K = 128 the 128-column ones, where both are bound by the vector ALU
+//     and q, k and e^g cost those fewer LDS reads (H = 16, 16 / 100 tokens: B = 24 28.7 / 26.6 and 130 / 115, B = 32
+//     30.5 / 33.9 and 132 / 145, B = 64 53.8 / 61.1 and 259 / 296); at K = 192 the scalar gate, whose decay costs those one
+//     multiplication by a register (GDN, H = 16, 100 tokens: B = 16 156 / 160, B = 31 276 / 309; KDA 176 / 144 and
+//     327 / 277).  At K = 32 and 64 the wide split stays ahead (B = 64, K = 64: 16 tokens 38.1 / 33.9, 100 tokens
+//     186 / 161).
+// A packed call is judged by its average sequence, the offsets being on the device: among many short sequences the recurrent
+// kernel is faster (H = 16, K = 128, 128 sequences of 4 tokens 51 / 91), but one long prompt among them takes it 0.95 us a
+// token (250 sequences of one token and one of 1,500: 1,421 / 922).
 hipError_t launch_sequential(const gdr_args& a, hipStream_t stream) {
   const int64_t n = a.cu_seqlens ? a.n_seqs : a.batch, columns = n * a.heads * a.value_dim;
   const int64_t tokens = a.cu_seqlens ? a.seq_len / n : a.seq_len;  // of an average sequence
-  const bool few = tokens < (a.key_dim > 128 && columns > 8192 ? 64 : 8);
-  const bool full = a.key_dim == 128 && a.value_dim % 128 == 0 && columns >= 65536;
+  const int enough = a.key_dim > 128 && columns > 8192 ? 64 : a.key_dim == 256 && columns > 4096 ? 16 : 8;
+  const bool few = tokens < enough;
+  const bool full = a.key_dim == 128   ? a.value_dim % 128 == 0 && columns >= 65536
+                    : a.key_dim == 192 ? a.variant == GDR_GDN && columns >= 32768
+                                       : false;
   if (few || full) return launch_recurrent(a, stream);
   return a.q.dtype == GDR_BF16 ? launch_t<__bf16>(a, stream) : launch_t<float>(a, stream);
 }
