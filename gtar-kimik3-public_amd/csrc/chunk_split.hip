@@ -303,8 +303,8 @@ __device__ __forceinline__ R input16(const void* p) {
 // f16 builds with a per-channel gate, whose diagonal strip tile carries extra bf16 operands (172 VGPRs for KDA; at 168
 // its spills cost more than the third workgroup gives, 274 -> 287 us at B = 2, T = 8,111), and the any-width
 // convolution, whose widest path holds 11 input rows and 8 weight rows per thread, are held to two so that they do not
-// spill.  kNT (plain
-// op only, bf16 or f16): the q, k, gate and V rows are loaded with the non-temporal hint (`use_nt_hint` below decides).
+// spill.  kNT (plain op only, bf16 or f16): the q, k, gate and V rows are loaded with the non-temporal hint
+// (`launch_prep_plain` below decides).
 template <int VARIANT, int K, int kPro = 0, int kNT = 0, typename T = __bf16>
 __global__ __launch_bounds__(256, ((__is_same(T, _Float16) && (VARIANT == GDR_KDA || VARIANT == GDR_GLA)) || (kPro & 16)) ? 2 : 3) void chunk_prep_kernel(const gdr_args a, int nc,
                                                                                          int64_t rec_bytes,
@@ -1389,6 +1389,11 @@ int64_t slots_per_head(const gdr_args& a) {
   return int64_t(a.batch) * ((a.seq_len + kChunk - 1) / kChunk);
 }
 
+template <int K>
+int64_t record_bytes(const gdr_args& a) {
+  return slots_per_head(a) * a.heads * Rec<K>::bytes(a.value_dim);
+}
+
 // Whether the call's single-use input rows (prep) and its outputs, states and u (scan) carry the non-temporal hint.
 // It pays when the records are about one to four times the 256 MB memory-side cache: the hint keeps inputs and
 // outputs from displacing the records the scan is about to read.  KDA at T = 4096, H = 16 (with the scan's output
@@ -1401,7 +1406,7 @@ int64_t slots_per_head(const gdr_args& a) {
 template <int K>
 bool use_nt_hint(const gdr_args& a) {
   constexpr int64_t kMin = int64_t(256) << 20, kMax = int64_t(1) << 30;
-  const int64_t records = slots_per_head(a) * a.heads * Rec<K>::bytes(a.value_dim);
+  const int64_t records = record_bytes<K>(a);
   if (records < kMin || records > kMax) return false;
   return (int64_t(a.seq_len) * a.out.stride_t + a.value_dim) * 4 < (int64_t(1) << 32);
 }
@@ -1419,11 +1424,20 @@ hipError_t launch_prep(const gdr_args& a, const gdr_prologue& pro, hipStream_t s
   return hipGetLastError();
 }
 
-// The plain op's prep, with the hinted input loads when the call asks for them.
+// The plain op's prep, with the hinted input loads where they pay.  f16 calls keep them to K = 128, value dims of 128 (GLA:
+// 128 up) and records up to 384 MiB (us per call without / with them, the scan's hints in both, H = 16: V = 128 KDA
+// B = 1, T = 16,000 404 / 376, GDN 388 / 360, GLA B = 4, T = 4,096 205 / 191; GLA V = 256 252 / 247); beyond, they cost
+// (KDA V = 128 B = 8, T = 5,000 515 / 530; V = 256 B = 4, T = 4,096 298 / 307; V = 64 B = 8, T = 8,000 698 / 738; K = V = 64
+// 428 / 446).
 template <int VARIANT, int K, typename T = __bf16>
 hipError_t launch_prep_plain(const gdr_args& a, hipStream_t stream) {
-  return use_nt_hint<K>(a) ? launch_prep<VARIANT, K, 0, T, 1>(a, gdr_prologue{}, stream)
-                           : launch_prep<VARIANT, K, 0, T>(a, gdr_prologue{}, stream);
+  constexpr bool kF16 = __is_same(T, _Float16);
+  if constexpr (!kF16 || K == 128) {
+    const bool pays = !kF16 || (record_bytes<K>(a) <= int64_t(384) << 20 &&
+                                (VARIANT == GDR_GLA ? a.value_dim >= 128 : a.value_dim == 128));
+    if (pays && use_nt_hint<K>(a)) return launch_prep<VARIANT, K, 0, T, 1>(a, gdr_prologue{}, stream);
+  }
+  return launch_prep<VARIANT, K, 0, T>(a, gdr_prologue{}, stream);
 }
 
 }  // namespace
