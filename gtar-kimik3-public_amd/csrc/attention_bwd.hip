@@ -25,7 +25,10 @@
 // SIMD, so what helps is less of everything in it: tile copies with one 32-bit lane offset instead of 64-bit address
 // arithmetic per copy, no mask selects in whole tiles, exponentials issued beside dP's MFMAs.  Measured (72,292 packed
 // tokens, 16 / 8 heads, D = 128, before -> after): dQ 1,445 -> 1,277 us, dK/dV 2,284 -> 2,069 us; D = 64 773 -> 700 and
-// 1,187 -> 1,150.  Tried for dK/dV and slower: 128-row tiles split over eight waves (2,337), two four-wave sets taking
+// 1,187 -> 1,150.  Sequences of one or two tiles pay 1 to 2 us per call for the exchange at the end and the spread of lse
+// and delta (33 tokens, D = 128, 16 / 8 heads: dK/dV 7.1 -> 9.3 us; 60 sequences of 64 24.0 -> 26.4; 300 tokens 53.4 ->
+// 52.6); the split by keys is not kept for them, because a packed sequence has to equal its own call bit for bit.  Tried
+// for dK/dV and slower: 128-row tiles split over eight waves (2,337), two four-wave sets taking
 // alternate tiles in one workgroup (2,397; faster only for a single long sequence, 179 against 217 us at 4,096 tokens).
 // Only tiles crossing the diagonal or the sequence end are masked.  No atomics: every output element has one
 // owning lane, so the result does not depend on scheduling.
