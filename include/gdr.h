@@ -347,7 +347,10 @@ int gdr_norm_gate_fwd(const gdr_norm_gate_args* args, hipStream_t stream);
 int gdr_norm_gate_rounded_fwd(const gdr_norm_gate_args* args, hipStream_t stream);
 
 /* The residual stream of the stack's blocks (src/models/kimi_k3.py:39-66 with RMSNorm src/layers/rmsnorm.py:11-16):
- * sum = residual + add in f32, out = bf16(weight * sum / sqrt(mean(sum^2) + eps)) over rows of `dim` values. */
+ * sum = residual + add in f32, out = bf16(weight * sum / sqrt(mean(sum^2) + eps)) over rows of `dim` values.
+ * A call holds what one launch does, fewer than 2^32 threads: here rows < 2^26, below tokens * heads < 2^28 (head norms)
+ * and rows * dim < 2^35 (SwiGLU; 2^32 where dim, stride or an address is not a multiple of 8 values); the norm-gate's
+ * B * T * H < 2^30.  (Each bound is one workgroup lower.)  More is GDR_ERR_UNSUPPORTED. */
 typedef struct gdr_add_norm_args {
   int32_t abi_version;    /* must equal GDR_ABI_VERSION */
   int32_t dim;            /* values per row */
