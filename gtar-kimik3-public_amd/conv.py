@@ -24,16 +24,28 @@ def _writable_in_place(state: torch.Tensor, dtype: torch.dtype) -> bool:
 def _span(t: torch.Tensor):
     """The addresses [first, end) that t's elements lie between (strides are not negative)."""
     first = t.data_ptr()
-    if t.numel() == 0:
-        return first, first
-    return first, first + t.element_size() * (1 + sum((n - 1) * s for n, s in zip(t.shape, t.stride())))
+    if t.is_contiguous():
+        return first, first + t.nbytes
+    last = 0
+    for n, stride in zip(t.shape, t.stride()):
+        if n == 0:
+            return first, first
+        last += (n - 1) * stride
+    return first, first + t.element_size() * (last + 1)
 
 
 def _apart(written, read) -> bool:
     """Whether no tensor that a kernel writes shares memory with another one or with one that it reads (None: absent)."""
     spans = sorted(map(_span, written))
-    return all(a[1] <= b[0] for a, b in zip(spans, spans[1:])) and \
-        all(a[1] <= b[0] or b[1] <= a[0] for a in spans for b in (_span(t) for t in read if t is not None))
+    if any(a[1] > b[0] for a, b in zip(spans, spans[1:])):
+        return False
+    first, end = spans[0][0], spans[-1][1]
+    for t in read:
+        if t is not None and t.data_ptr() < end:
+            low, high = _span(t)
+            if high > first and any(low < s[1] and s[0] < high for s in spans):
+                return False
+    return True
 
 
 def short_convolution(
